@@ -15,6 +15,7 @@
 // accumulators and the reference's f32 group order. The f32 steps around them follow the
 // reference's order: the mean is a sequential sum per channel, the exponentials' sum is the
 // scalar backend's (eight offset sums over whole runs of eight, then the rest and those sums).
+#include "attention.h"
 #include "common.h"
 #include "proj.h"
 
@@ -30,21 +31,6 @@ constexpr int kMaxRowBytes = 64 * 1024;  // one padded score row in LDS: at most
 constexpr int kMaxHeadDim = 1024;
 
 size_t pad32(size_t n) { return (n + 31) / 32 * 32; }
-
-// exp_fast (ops.rs:137-153): clamped below at EXP_MIN, n = round(x · log2 e) ties to even,
-// r = fma(−n, ln 2, x), the degree-4 Taylor polynomial in fused multiply-adds, times 2^n.
-__device__ __forceinline__ float ref_exp_fast(float x)
-{
-    x = fmaxf(x, -87.0f);
-    const float n = rintf(x * 1.44269504088896340736f);
-    const float r = __builtin_fmaf(-n, 0.693147180559945309417f, x);
-    float poly = 1.0f / 24.0f;
-    poly = __builtin_fmaf(poly, r, 1.0f / 6.0f);
-    poly = __builtin_fmaf(poly, r, 0.5f);
-    poly = __builtin_fmaf(poly, r, 1.0f);
-    poly = __builtin_fmaf(poly, r, 1.0f);
-    return poly * __int_as_float((int(n) + 127) << 23);
-}
 
 // keyT[(t · hd + d) · kpad + k] = key[k][d] of table t = image · kv_heads + kh: the keys of every
 // (image, key head) with channels as rows, through 64 x 64 tiles in LDS (both sides coalesced).
@@ -117,20 +103,6 @@ __device__ __forceinline__ void clear_block(int8_t *codes32, float *scale)
     dst[0] = make_int4(v, v, v, v);
     dst[1] = make_int4(v, v, v, v);
     *scale = 0.0f;
-}
-
-// Q7b32 levels of four values at scale d (quant.rs:143-150: rne(x / d) clamped to ±63 through the
-// saturating cast), packed as one dword of device levels.
-__device__ __forceinline__ int q7_levels4(const float (&x)[4], float d)
-{
-    int l[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const float v = __builtin_rintf(x[j] / d);
-        const int level = v != v ? 0 : v >= 127.0f ? 127 : v <= -128.0f ? -128 : int(v);
-        l[j] = level < -63 ? -63 : (level > 63 ? 63 : level);
-    }
-    return pack4(l[0], l[1], l[2], l[3]);
 }
 
 // Scratch::quantize's key matrices (attention.rs:100-118) for every (image, key head) at once:
@@ -545,6 +517,17 @@ int run(const fg_attention *c, float *out, hipStream_t st, const Shape &s, const
     return FG_OK;
 }
 
+// Whether the call runs in the one launch of attention_fused.hip instead of a unit at a time.
+bool takes_fused(const fg_attention *c)
+{
+    if (c->head_dim > 128 || getenv("FG_ATTEND_UNITS")) return false;
+    // its kernels count lanes and query tiles in 32 bits
+    const size_t tables = c->images * c->kv_heads, blocks = (c->keys + 31) / 32;
+    const size_t lanes = std::max({tables * blocks * 32 * 8 * ((c->head_dim + 31) / 32), tables * blocks * (c->head_dim + 8),
+                                   c->images * c->heads * ((c->queries + 127) / 128) * 256});
+    return lanes < (size_t(1) << 31);
+}
+
 }  // namespace
 }  // namespace fg
 
@@ -576,11 +559,12 @@ extern "C" int fg_attend(const fg_attention *c, float *out, void *stream)
                                    s.qtables * s.queries * (s.pd / 4), s.qtables * s.queries * s.hd});
     if (lanes >= (size_t(1) << 31)) return set_error(FG_ERR_SHAPE, "fg_attend: at most 2^31 - 1 values of queries, keys or outputs");
     const hipStream_t st = static_cast<hipStream_t>(stream);
+    const bool fused = takes_fused(c);
     Scratch w(s);
     void *ws = nullptr;
-    FG_HIP(workspace_alloc(&ws, w.total(), st));
+    FG_HIP(workspace_alloc(&ws, fused ? attend_fused_bytes(c) : w.total(), st));
     w.carve(ws);
-    int rc = run(c, out, st, s, w);
+    int rc = fused ? launch_attend_fused(c, out, ws, st) : run(c, out, st, s, w);
     // the scratch goes back to the pool in stream order, after the call's last kernel
     const hipError_t e = hipFreeAsync(ws, st);
     if (rc == FG_OK && e != hipSuccess) rc = check_hip(e, "hipFreeAsync");
