@@ -517,15 +517,29 @@ int run(const fg_attention *c, float *out, hipStream_t st, const Shape &s, const
     return FG_OK;
 }
 
-// Whether the call runs in the one launch of attention_fused.hip instead of a unit at a time.
+// Whether the call runs in the one launch of attention_fused.hip instead of a unit at a time. The
+// one launch walks a row's blocks of 32 keys in order, so few rows over many keys leave the chip
+// idle behind that chain; a unit at a time pays two launches per unit but spreads its keys. Both
+// sides as fitted, in microseconds, to measurements over 1 to 48 units, 1 to 1024 queries, 64 to
+// 16384 keys and heads of 32 to 128, of which the line misplaces those within about 20 % of it
+// (fast exponentials, heads of 64, one launch against unit by unit: 6 units x 1024 queries x 1024
+// keys 76 against 109; 1 unit of the same 75 against 56; 12 units x 1024 x 4096 256 against 371;
+// 12 units x 1 x 4096 249 against 210).
 bool takes_fused(const fg_attention *c)
 {
+    // FG_ATTEND_UNITS sizes the step-by-step batches, so it asks for them
     if (c->head_dim > 128 || getenv("FG_ATTEND_UNITS")) return false;
     // its kernels count lanes and query tiles in 32 bits
     const size_t tables = c->images * c->kv_heads, blocks = (c->keys + 31) / 32;
     const size_t lanes = std::max({tables * blocks * 32 * 8 * ((c->head_dim + 31) / 32), tables * blocks * (c->head_dim + 8),
                                    c->images * c->heads * ((c->queries + 127) / 128) * 256});
-    return lanes < (size_t(1) << 31);
+    if (lanes >= (size_t(1) << 31)) return false;
+    const double units = double(c->images * c->heads), keys = double(c->keys), queries = double(c->queries);
+    const double hd = double(c->head_dim), waves = units * std::ceil(queries / 32);
+    const double block = 0.65 + 0.0215 * hd + (c->exponentials == FG_EXP_FAST ? 0.0 : 0.5);
+    const double fused = 20 + double(blocks) * block * std::max(1.0, 0.7 * waves / 1024);
+    const double steps = 45 + 6.6 * units + 1.2e-4 * keys * hd + units * keys * (0.00115 + 3.5e-6 * queries);
+    return fused <= steps;
 }
 
 }  // namespace

@@ -22,8 +22,12 @@
 // [32 channels][half][channel][16 keys in the lane's order], value scales [channel]. A workgroup
 // of four waves (128 queries) brings two records at a time into LDS, double-buffered.
 //
-// Bound: VALU issue (about 55 operations a score with 72 channels, 250 us for 16 heads of
-// 4096 x 4096 at the measured 2.3 cycles each) beside the matrix cores' 35 us.
+// Bound: instruction issue. Additions and multiplications take 2.4 cycles a wave with two waves on the
+// SIMD, fused multiply-adds, maxima and byte permutes 4.2, so totals are converted by subtraction
+// (unbiased) and exponents taken from an addition's low bits (ref_exp): 4096 x 4096, 16 heads of
+// 72, in 321 us (409 with conversion instructions), 365 a call with the keys' and values'
+// preparation, against 941 unit by unit. 16 queries a wave (16 x 16 products, four waves a SIMD)
+// take 530 us: the same arithmetic with twice the instructions around it.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -65,56 +69,68 @@ struct FusedParams {
     float scale;
 };
 
-constexpr int kMeanThreads = 1024, kMeanKeys = 256;
+constexpr int kMeanThreads = 256, kMeanChannels = 16, kMeanKeys = 512;
 
 // The keys' mean (attention.rs:104-110): per channel of an image's key row a sum over the keys in
-// order. A workgroup takes 64 neighbouring channels: its sixteen waves bring 256 keys at a time
-// into LDS (the next 256 in flight), and a lane of the first wave adds each channel's.
+// order. A workgroup takes 16 neighbouring channels: its waves bring 512 keys at a time into LDS, a
+// thread four neighbouring keys of a channel as one 16-byte run, with the next two chunks in
+// flight, and a lane of the first wave adds each channel's. The chain of additions (2.8 ns each) is
+// the bound, as long as enough CUs share the reading: 4096 keys of 1152 channels 25 us in 72
+// workgroups, of which the chain is 11.5 (30 us in 18 workgroups of 64 channels: about 50 GB/s a CU).
 __device__ __forceinline__ void key_means(const FusedParams &p, int image, int c0)
 {
-    extern __shared__ __align__(16) float chunk[];  // [2][kMeanKeys][64]
-    const int width = p.kv_heads * p.hd, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const float *src = p.key + size_t(image) * size_t(p.keys) * p.key_stride + p.key_offset + min(c0 + lane, width - 1);
-    constexpr int kLoads = kMeanKeys / 16;
-    float r[kLoads];
-    auto load = [&](int k0) {
-#pragma unroll
-        for (int u = 0; u < kLoads; u++) r[u] = src[size_t(min(k0 + wave + 16 * u, p.keys - 1)) * p.key_stride];
-    };
-    load(0);
+    extern __shared__ __align__(16) v4f chunk[];  // [2][kMeanKeys / 4][kMeanChannels]
+    constexpr int C = kMeanChannels, kSlots = kMeanThreads / C;
+    constexpr int kRuns = kMeanKeys / 4 / kSlots;  // runs of four keys a thread brings of a chunk
+    const int width = p.kv_heads * p.hd, channel = threadIdx.x % C, slot = threadIdx.x / C;
+    const float *src = p.key + size_t(image) * size_t(p.keys) * p.key_stride + p.key_offset + min(c0 + channel, width - 1);
     float s = 0.0f;
-    int at = 0;
-    for (int k0 = 0; k0 < p.keys; k0 += kMeanKeys, at ^= 1) {
-        float *buf = chunk + at * kMeanKeys * 64;
+    auto load = [&](v4f (&r)[kRuns], int k0) {
 #pragma unroll
-        for (int u = 0; u < kLoads; u++) buf[(wave + 16 * u) * 64 + lane] = r[u];
-        __syncthreads();
-        if (k0 + kMeanKeys < p.keys) load(k0 + kMeanKeys);
-        if (wave == 0) {
-            // runs of 32 keys in two register sets in turn: a run's reads go out before the
-            // additions of the one before it
-            const int n = min(kMeanKeys, p.keys - k0), runs = n / 32;
-            float x[2][32];
-            auto fetch = [&](float (&v)[32], int run) {
+        for (int u = 0; u < kRuns; u++) {
 #pragma unroll
-                for (int u = 0; u < 32; u++) v[u] = buf[(run * 32 + u) * 64 + lane];
-                __builtin_amdgcn_sched_barrier(0);
-            };
-            auto add = [&](const float (&v)[32]) {
-#pragma unroll
-                for (int u = 0; u < 32; u++) s = s + v[u];
-            };
-            if (runs > 0) fetch(x[0], 0);
-            for (int run = 0; run < runs; run += 2) {
-                fetch(x[1], min(run + 1, runs - 1));
-                add(x[0]);
-                fetch(x[0], min(run + 2, runs - 1));
-                if (run + 1 < runs) add(x[1]);
-            }
-            for (int k = runs * 32; k < n; k++) s = s + buf[k * 64 + lane];
+            for (int e = 0; e < 4; e++) r[u][e] = src[size_t(min(k0 + 4 * (slot + kSlots * u) + e, p.keys - 1)) * p.key_stride];
         }
+    };
+    auto step = [&](v4f (&r)[kRuns], int k0, v4f *buf) {
+#pragma unroll
+        for (int u = 0; u < kRuns; u++) buf[(slot + kSlots * u) * C + channel] = r[u];
+        __syncthreads();
+        if (k0 + 2 * kMeanKeys < p.keys) load(r, k0 + 2 * kMeanKeys);
+        if (threadIdx.x >= C) return;
+        // runs of 32 keys in two register sets in turn: a run's reads go out before the additions of
+        // the one before it
+        const int n = min(kMeanKeys, p.keys - k0), runs = n / 32;
+        v4f x[2][8];
+        auto fetch = [&](v4f (&v)[8], int run) {
+#pragma unroll
+            for (int u = 0; u < 8; u++) v[u] = buf[(run * 8 + u) * C + channel];
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto add = [&](const v4f (&v)[8]) {
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) s = s + v[u][e];
+            }
+        };
+        if (runs > 0) fetch(x[0], 0);
+        for (int run = 0; run < runs; run += 2) {
+            fetch(x[1], min(run + 1, runs - 1));
+            add(x[0]);
+            fetch(x[0], min(run + 2, runs - 1));
+            if (run + 1 < runs) add(x[1]);
+        }
+        for (int k = runs * 32; k < n; k++) s = s + buf[k / 4 * C + channel][k % 4];
+    };
+    v4f even[kRuns], odd[kRuns];
+    load(even, 0);
+    load(odd, kMeanKeys);
+    for (int k0 = 0; k0 < p.keys; k0 += 2 * kMeanKeys) {
+        step(even, k0, chunk);
+        if (k0 + kMeanKeys < p.keys) step(odd, k0 + kMeanKeys, chunk + kMeanKeys / 4 * C);
     }
-    if (wave == 0 && c0 + lane < width) p.mean[size_t(image) * width + c0 + lane] = s / float(p.keys);
+    if (slot == 0 && c0 + channel < width) p.mean[size_t(image) * width + c0 + channel] = s / float(p.keys);
 }
 
 // The values' half of the records (Scratch::transpose, attention.rs:119-137): one thread per
@@ -158,7 +174,7 @@ __global__ __launch_bounds__(kMeanThreads) void mean_and_values_kernel(FusedPara
 {
     const int b = int(blockIdx.x);
     if (b < mean_blocks) {
-        key_means(p, b / mean_groups, b % mean_groups * 64);
+        key_means(p, b / mean_groups, b % mean_groups * kMeanChannels);
         return;
     }
     value_record<PB, TJ>(p, unsigned(b - mean_blocks) * kMeanThreads + threadIdx.x, values);
@@ -293,14 +309,14 @@ __global__ __launch_bounds__(256, 2) void attend_fused_kernel(FusedParams p)
     }
 
     // two records (their first `bytes` bytes) from global memory to registers, then to LDS
-    int4 staged[kRounds];
+    v4i staged[kRounds];
     auto load = [&](int stage, int bytes) {
         const int per = bytes / 16;
 #pragma unroll
         for (int r = 0; r < kRounds; r++) {
             const int i = min(tid + 256 * r, 2 * per - 1), second = i >= per;
             const int kb = min(2 * stage + second, p.nkb - 1);
-            staged[r] = reinterpret_cast<const int4 *>(records + size_t(kb) * R::kBytes)[i - second * per];
+            staged[r] = reinterpret_cast<const v4i *>(records + size_t(kb) * R::kBytes)[i - second * per];
         }
     };
     auto store = [&](int at, int bytes) {
@@ -308,9 +324,12 @@ __global__ __launch_bounds__(256, 2) void attend_fused_kernel(FusedParams p)
 #pragma unroll
         for (int r = 0; r < kRounds; r++) {
             const int i = tid + 256 * r, second = i >= per;
-            if (i < 2 * per) reinterpret_cast<int4 *>(buffers[at] + second * R::kBytes)[i - second * per] = staged[r];
+            if (i < 2 * per) reinterpret_cast<v4i *>(buffers[at] + second * R::kBytes)[i - second * per] = staged[r];
         }
     };
+    // both of a stage's blocks at once where their registers allow
+    constexpr bool kTogether = PB < 4 && !(PB == 3 && TJ == 3);
+    const v16i biased = biased_zero<v16i>();
     // N blocks' scores before their scaling, the reference's order over the channel blocks (its
     // first addition, to +0, is left out: a term of -0 gives the same exponential). The scale
     // products of two (key block, channel block) pairs come from one f32 outer product
@@ -318,7 +337,6 @@ __global__ __launch_bounds__(256, 2) void attend_fused_kernel(FusedParams p)
     // LDS read per lane where the scales in the product's layout are four of 16 bytes.
     auto scores = [&](const char *rec, auto count, auto &s) {
         constexpr int N = decltype(count)::value, F = N * PB;
-        const v16i zero = {};
         const v32f zero32 = {};
 #pragma unroll
         for (int f = 0; f < F; f += 2) {
@@ -331,10 +349,10 @@ __global__ __launch_bounds__(256, 2) void attend_fused_kernel(FusedParams p)
                 if (f + e >= F) break;
                 const int n = (f + e) / PB, b = (f + e) % PB;
                 const v4i k = *reinterpret_cast<const v4i *>(rec + n * R::kBytes + b * 1024 + lane * 16);
-                const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(k, ql[b], zero, 0, 0, 0);
+                const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(k, ql[b], biased, 0, 0, 0);
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
-                    const float term = float(d[r]) * scale[16 * e + r];
+                    const float term = unbiased(d[r]) * scale[16 * e + r];
                     s[n][r] = b == 0 ? term : s[n][r] + term;
                 }
             }
@@ -421,13 +439,12 @@ __global__ __launch_bounds__(256, 2) void attend_fused_kernel(FusedParams p)
         // their scale products as the scores': whole tiles of 32 channels by outer products, two to
         // one, a short last tile by multiplications
         constexpr int W = TJ > 2 ? PB : PB - 1, F = N * W;
-        const v16i zero = {};
         const v32f zero32 = {};
         auto dots = [&](int n, int c) {
             const int rows = c == PB - 1 ? 8 * TJ : 32;
             const char *values = rec + n * R::kBytes + R::kValues + c * 1024;
             const v4i v = *reinterpret_cast<const v4i *>(values + (half * rows + min(l31, rows - 1)) * 16);
-            return __builtin_amdgcn_mfma_i32_32x32x32_i8(v, levels[n], zero, 0, 0, 0);
+            return __builtin_amdgcn_mfma_i32_32x32x32_i8(v, levels[n], biased, 0, 0, 0);
         };
 #pragma unroll
         for (int f = 0; f < F; f += 2) {
@@ -444,7 +461,7 @@ __global__ __launch_bounds__(256, 2) void attend_fused_kernel(FusedParams p)
                 const int n = (f + e) / max(W, 1), c = (f + e) % max(W, 1);
                 const v16i t = dots(n, c);
 #pragma unroll
-                for (int r = 0; r < (c == PB - 1 ? 4 * TJ : 16); r++) acc[c][r] = acc[c][r] + float(t[r]) * scale[16 * e + r];
+                for (int r = 0; r < (c == PB - 1 ? 4 * TJ : 16); r++) acc[c][r] = acc[c][r] + unbiased(t[r]) * scale[16 * e + r];
             }
         }
         if (W < PB) {
@@ -455,7 +472,7 @@ __global__ __launch_bounds__(256, 2) void attend_fused_kernel(FusedParams p)
                 for (int j = 0; j < TJ; j++) {
                     const v4f vs = *reinterpret_cast<const v4f *>(rec + n * R::kBytes + R::kValueScales + (32 * (PB - 1) + 8 * j + 4 * half) * 4);
 #pragma unroll
-                    for (int i = 0; i < 4; i++) acc[PB - 1][4 * j + i] = acc[PB - 1][4 * j + i] + float(t[4 * j + i]) * (vs[i] * d[n]);
+                    for (int i = 0; i < 4; i++) acc[PB - 1][4 * j + i] = acc[PB - 1][4 * j + i] + unbiased(t[4 * j + i]) * (vs[i] * d[n]);
                 }
             }
         }
@@ -468,7 +485,12 @@ __global__ __launch_bounds__(256, 2) void attend_fused_kernel(FusedParams p)
         if (!active) continue;
         const char *buf = buffers[st & 1];
         if (st < pairs) {
-            weigh(buf, Two{}, std::false_type{}, 64);
+            if (kTogether) {
+                weigh(buf, Two{}, std::false_type{}, 64);
+            } else {
+#pragma unroll 1
+                for (int blk = 0; blk < 2; blk++) weigh(buf + blk * R::kBytes, One{}, std::false_type{}, 32);
+            }
         } else {
             for (int blk = 0; blk < 2 && 2 * st + blk < p.nkb; blk++)
                 weigh(buf + blk * R::kBytes, One{}, std::true_type{}, p.keys - 32 * (2 * st + blk));
@@ -517,11 +539,9 @@ int launch_as(FusedParams p, int images, bool fast, hipStream_t s)
 {
     using R = Record<PB, TJ>;
     const int tables = images * p.kv_heads;
-    const int groups = (p.kv_heads * p.hd + 63) / 64, means = images * groups;
+    const int groups = (p.kv_heads * p.hd + kMeanChannels - 1) / kMeanChannels, means = images * groups;
     const unsigned values = unsigned(tables) * unsigned(p.nkb) * unsigned(R::kChannels);
-    const size_t lds = size_t(2) * kMeanKeys * 64 * 4;
-    FG_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(mean_and_values_kernel<PB, TJ>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+    const size_t lds = size_t(2) * kMeanKeys * kMeanChannels * 4;
     mean_and_values_kernel<PB, TJ><<<unsigned(means) + (values + kMeanThreads - 1) / kMeanThreads, kMeanThreads, lds, s>>>(
         p, means, groups, values);
     FG_HIP(hipGetLastError());
