@@ -564,6 +564,259 @@ __global__ __launch_bounds__(kAttnThreads) void attn_rows_kernel(AttnParams a, i
     }
 }
 
+// A prefill's attention in parallel order on the matrix cores, for head sizes 32, 64 and 128: flash
+// attention in f32 (v_mfma_f32_32x32x2_f32, products and sums no less exact than the VALU's). A
+// workgroup of eight waves takes 32 rows of one query head; wave w takes the blocks of 32 keys w,
+// w + 8, ... with a running maximum, total and weighted values of its own, merged through LDS at the
+// end, and the rows' outputs are quantized per group of 32 for the output projection.
+//   scores: formed transposed (keys x rows), so lane l holds row l % 32 against keys
+//           8j + 4(l / 32) + i in register 4j + i. The two operands agree on which dimensions a step
+//           takes (half l / 32 holds dimensions (l / 32)·D/2 on), so a lane reads whole runs of its
+//           key's row and keeps its query's in registers;
+//   weights: ops::exp of the scores less the running maximum; a row's sixteen values in each of
+//           its two lanes, so its maximum and total take one lane swap;
+//   values: the weights are the second operand in place: step (j, i) takes keys 8j + i and 8j + 4 + i,
+//           whose values the first operand reads as rows of 32 neighbouring dimensions.
+// The chunk's keys and values are in the caches before the launch (keep_rows_kernel). Every row is
+// masked past its own position (Mask::Causal); a masked weight is 0, which a non-finite value of a
+// later row would still turn into NaN, so a block that holds one adds its keys singly and only to
+// the rows that see them.
+// Bound: the f32 matrix rate, 4096 cycles a block of 32 rows x 32 keys x 64 dimensions, beside about
+// 1300 of VALU work; with few blocks a wave, the chain of loads before and merge after them. 14 heads
+// of 64 over 2, 512 rows, after 0, 512 and 1024 others: 30 us a chunk on average where the VALU
+// kernel below (each row of the block reading every staged key and value) took 163; 158 rows 11.1
+// and 3.2 for keep_rows_kernel where it took 17.5.
+constexpr int kFlashRows = 32, kFlashWaves = 8;
+
+template <int D>
+constexpr int flash_stride() { return D + 4; }  // a row's partial outputs in LDS: 16-byte rows on different banks
+template <int D>
+constexpr size_t flash_smem() { return size_t(kFlashWaves) * kFlashRows * (flash_stride<D>() + 2) * 4; }
+
+template <int D>
+__global__ __launch_bounds__(64 * kFlashWaves, 2) void attn_flash_kernel(AttnParams a, int n)
+{
+    typedef float v16f __attribute__((ext_vector_type(16)));
+    extern __shared__ __align__(16) float ash[];
+    constexpr int H = D / 2, T = D / 32, S = flash_stride<D>();
+    float *part = ash;                                     // [wave][row][S]
+    float *tops = part + kFlashWaves * kFlashRows * S;     // [wave][row] maxima
+    float *tots = tops + kFlashWaves * kFlashRows;         // [wave][row] totals
+    const int head = blockIdx.x, z0 = int(gridDim.y - 1 - blockIdx.y) * kFlashRows;  // the longest rows first
+    const int kv = head / (a.heads / a.kv_heads);
+    const int tid = threadIdx.x, lane = tid & 63, l31 = lane & 31, half = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const float *kbase = a.kcache + a.layer_base + size_t(kv) * a.capacity * D;
+    const float *vbase = a.vcache + a.layer_base + size_t(kv) * a.capacity * D;
+    const int first = a.keys - 1, rows = min(kFlashRows, n - z0);
+    const int position = first + z0 + min(l31, rows - 1);  // this lane's row (the last again past the rows)
+    const int seen = first + z0 + rows;                    // keys the block's last row sees
+    const int blocks = (seen + 31) / 32;
+
+    // the block's queries, rotated by halves at their positions (ops.rs:77-85) by the first waves, then
+    // every lane's row, this half's dimensions. (Read by the lanes that need them, the rows would
+    // cost each wave a cache line per lane and load.)
+    for (int e = tid; e < kFlashRows * (D / 8); e += 64 * kFlashWaves) {
+        const int r = e / (D / 8), c = (e - r * (D / 8)) * 4, z = z0 + min(r, rows - 1);
+        const float *src = a.qkv + size_t(z) * a.qkv_stride + size_t(head) * D + c;
+        const float *cs = a.rope + size_t(first + z) * D + c;
+        const v4f x = *reinterpret_cast<const v4f *>(src), y = *reinterpret_cast<const v4f *>(src + H);
+        const v4f co = *reinterpret_cast<const v4f *>(cs), si = *reinterpret_cast<const v4f *>(cs + H);
+        *reinterpret_cast<v4f *>(part + r * S + c) = x * co - y * si;
+        *reinterpret_cast<v4f *>(part + r * S + c + H) = y * co + x * si;
+    }
+    __syncthreads();
+    v4f q[H / 4];
+#pragma unroll
+    for (int c = 0; c < H / 4; c++) q[c] = *reinterpret_cast<const v4f *>(part + l31 * S + half * H + 4 * c);
+    __syncthreads();  // the region is the waves' keys from here on
+    const float scale = 1.0f / sqrtf(float(D));
+    float top = -INFINITY, total = 0.0f;
+    v16f acc[T];
+#pragma unroll
+    for (int t = 0; t < T; t++) acc[t] = v16f{};
+    // a block's keys: whole rows by neighbouring lanes, then through this wave's part of LDS, a row
+    // per lane
+    float *const keys = part + wave * kFlashRows * S;
+    constexpr int kLoads = 32 * D / 256, kLanes = D / 4;  // 16-byte loads a lane, lanes a row
+    v4f k[kLoads];
+    auto load_keys = [&](int b) {
+#pragma unroll
+        for (int c = 0; c < kLoads; c++) {
+            const int r = c * (64 / kLanes) + lane / kLanes;
+            k[c] = *reinterpret_cast<const v4f *>(kbase + size_t(min(b * 32 + r, seen - 1)) * D + lane % kLanes * 4);
+        }
+    };
+    auto store_keys = [&]() {
+#pragma unroll
+        for (int c = 0; c < kLoads; c++)
+            *reinterpret_cast<v4f *>(keys + (c * (64 / kLanes) + lane / kLanes) * S + lane % kLanes * 4) = k[c];
+    };
+    // a block's values of 32 dimensions, in the operand's order
+    auto load_values = [&](int b, int t, float (&v)[16]) {
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+            v[r] = vbase[size_t(min(b * 32 + 8 * (r / 4) + 4 * half + r % 4, seen - 1)) * D + l31 + 32 * t];
+    };
+    // heads of 128 hold twice the query and sums: their keys and values are not loaded ahead
+    constexpr bool kAhead = D < 128;
+    if (kAhead && wave < blocks) load_keys(wave);
+    for (int b = wave; b < blocks; b += kFlashWaves) {
+        float v[kAhead ? T : 1][16];
+        if (kAhead) {
+#pragma unroll
+            for (int t = 0; t < T; t++) load_values(b, t, v[t]);
+            __builtin_amdgcn_sched_barrier(0);  // the values' loads stay ahead of the scores' products
+        } else {
+            load_keys(b);
+        }
+        store_keys();
+        v16f s = {};
+#pragma unroll
+        for (int c = 0; c < H / 4; c++) {
+            const v4f kc = *reinterpret_cast<const v4f *>(keys + l31 * S + half * H + 4 * c);
+#pragma unroll
+            for (int e = 0; e < 4; e++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kc[e], q[c][e], s, 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (kAhead && b + kFlashWaves < blocks) load_keys(b + kFlashWaves);
+        const bool edge = b * 32 + 31 > first + z0;  // some row does not see the block's last key
+        const int limit = position - b * 32;         // this row sees the block's keys 0..limit
+        float m = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            s[r] = s[r] * scale;
+            if (edge) s[r] = 8 * (r / 4) + 4 * half + r % 4 <= limit ? s[r] : -INFINITY;
+            m = fmaxf(m, s[r]);
+        }
+        const float2 mh = half_pair(m);
+        m = fmaxf(fmaxf(mh.x, mh.y), top);
+        const float base = m == -INFINITY ? 0.0f : m;  // every score so far -inf
+        const float shrink = ref_exp(top - base);
+        top = m;
+        float sum = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            float e = ref_exp(s[r] - base);
+            if (edge) e = 8 * (r / 4) + 4 * half + r % 4 <= limit ? e : 0.0f;
+            s[r] = e;
+            sum = sum + e;
+        }
+        const float2 sh = half_pair(sum);
+        total = total * shrink + (sh.x + sh.y);
+#pragma unroll
+        for (int t = 0; t < T; t++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[t][r] = acc[t][r] * shrink;
+#pragma unroll
+        for (int t = 0; t < T; t++) {
+            float(&vt)[16] = v[kAhead ? t : 0];
+            if (!kAhead) load_values(b, t, vt);
+            bool odd = false;  // a value that is not finite, in a block some row sees in part
+            if (edge) {
+                float x = 0.0f;
+#pragma unroll
+                for (int r = 0; r < 16; r++) x = x + vt[r] * 0.0f;  // NaN if any is infinite or NaN
+                odd = x != 0.0f;
+            }
+            if (!__any(odd)) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(vt[r], s[r], acc[t], 0, 0, 0);
+                continue;
+            }
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+#pragma unroll
+                for (int g = 0; g < 2; g++) {
+                    const int key = 8 * (r / 4) + 4 * g + r % 4;
+                    const v16f one = __builtin_amdgcn_mfma_f32_32x32x2f32(half == g ? vt[r] : 0.0f, half == g ? s[r] : 0.0f, v16f{}, 0, 0, 0);
+#pragma unroll
+                    for (int e = 0; e < 16; e++) acc[t][e] = key <= limit ? acc[t][e] + one[e] : acc[t][e];
+                }
+            }
+        }
+    }
+    // the waves' partial rows merged
+    {
+        float *dst = part + (wave * kFlashRows + l31) * S;
+#pragma unroll
+        for (int t = 0; t < T; t++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                *reinterpret_cast<v4f *>(dst + 32 * t + 8 * j + 4 * half) =
+                    v4f{acc[t][4 * j], acc[t][4 * j + 1], acc[t][4 * j + 2], acc[t][4 * j + 3]};
+        if (half == 0) {
+            tops[wave * kFlashRows + l31] = top;
+            tots[wave * kFlashRows + l31] = total;
+        }
+    }
+    __syncthreads();
+    const int live = min(kFlashWaves, blocks);  // waves that took keys
+    for (int e = tid; e < kFlashRows * (D / 4); e += 64 * kFlashWaves) {  // whole waves: D / 4 >= 8 lanes a row
+        const int r = e / (D / 4), c = (e - r * (D / 4)) * 4, sub = tid & 7;
+        float m = -INFINITY;
+        for (int w = 0; w < live; w++) m = fmaxf(m, tops[w * kFlashRows + r]);
+        float sum = 0.0f;
+        v4f x = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int w = 0; w < live; w++) {
+            const float f = ref_exp(tops[w * kFlashRows + r] - m);
+            const v4f y = *reinterpret_cast<const v4f *>(part + (w * kFlashRows + r) * S + c);
+            sum = sum + f * tots[w * kFlashRows + r];
+#pragma unroll
+            for (int i = 0; i < 4; i++) x[i] = x[i] + f * y[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) x[i] = x[i] / sum;
+        float amax = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
+        amax = max8(fmaxf(0.0f, amax));
+        int l0, l1, l2, l3;
+        const float d = scale_and_levels(amax, x[0], x[1], x[2], x[3], l0, l1, l2, l3);
+        const int levels = sum8(l0 + l1 + l2 + l3);
+        if (r >= rows) continue;
+        const size_t G = (size_t(z0 + r) * a.row_width + size_t(head) * D + c) / 32;
+        reinterpret_cast<int *>(a.q)[G * 8 + sub] = pack4(l0, l1, l2, l3);
+        if (sub == 0) {
+            a.scales[G] = d;
+            a.corr[G] = -a.zp * levels;
+        }
+    }
+}
+
+// A prefill chunk's keys rotated by halves at their positions, and its values, into the caches
+// (KvCache::keep, transformer.rs:166-180): a thread per (row, KV head, four pairs of dimensions).
+__global__ __launch_bounds__(256) void keep_rows_kernel(AttnParams a, int n)
+{
+    const int D = a.D, half = D / 2, per = D / 8;
+    const unsigned id = blockIdx.x * 256u + threadIdx.x;
+    if (id >= unsigned(n) * unsigned(a.kv_heads * per)) return;
+    const int j = int(id % unsigned(per)) * 4, kv = int(id / unsigned(per) % unsigned(a.kv_heads)), r = int(id / unsigned(per * a.kv_heads));
+    const int position = a.keys - 1 + r;
+    const float *key = a.qkv + size_t(r) * a.qkv_stride + size_t(a.heads + kv) * D + j;
+    const float *value = key + size_t(a.kv_heads) * D;
+    const float *cs = a.rope + size_t(position) * D + j;
+    const size_t at = a.layer_base + (size_t(kv) * a.capacity + size_t(position)) * D + j;
+    const v4f x = *reinterpret_cast<const v4f *>(key), y = *reinterpret_cast<const v4f *>(key + half);
+    const v4f c = *reinterpret_cast<const v4f *>(cs), s = *reinterpret_cast<const v4f *>(cs + half);
+    *reinterpret_cast<v4f *>(a.kkeep + at) = x * c - y * s;
+    *reinterpret_cast<v4f *>(a.kkeep + at + half) = y * c + x * s;
+    *reinterpret_cast<v4f *>(a.vkeep + at) = *reinterpret_cast<const v4f *>(value);
+    *reinterpret_cast<v4f *>(a.vkeep + at + half) = *reinterpret_cast<const v4f *>(value + half);
+}
+
+template <int D>
+int launch_flash(const AttnParams &a, int n, hipStream_t s)
+{
+    const unsigned threads = unsigned(n) * unsigned(a.kv_heads * (D / 8));
+    keep_rows_kernel<<<(threads + 255) / 256, 256, 0, s>>>(a, n);
+    FG_HIP(hipGetLastError());
+    constexpr size_t smem = flash_smem<D>();
+    if (smem > 64 * 1024)
+        FG_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(attn_flash_kernel<D>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   int(smem)));
+    attn_flash_kernel<D><<<dim3(unsigned(a.heads), unsigned((n + kFlashRows - 1) / kFlashRows)), 64 * kFlashWaves, smem, s>>>(a, n);
+    return FG_OK;
+}
+
 // LDS of attn_rows_kernel for a prefill whose last row sees kmax keys (0 when it does not fit 64 KiB
 // or the head is wider than a workgroup).
 inline size_t attn_rows_smem(int D, int kmax)
@@ -572,6 +825,20 @@ inline size_t attn_rows_smem(int D, int kmax)
     if (R < 1) return 0;
     const size_t bytes = (size_t(R) * ((kmax + 3) / 4 * 4) + size_t(4096 / D) * (D + 1) + size_t(R) * D + 16) * 4;
     return bytes <= 64 * 1024 ? bytes : 0;
+}
+
+// Which kernels a chunk of n rows whose last sees kmax keys takes, in parallel order (head sizes are
+// 32, 64 or 128). Four layers' reads with attn_flash_kernel against the others, microseconds:
+//   few keys, one launch instead of two: 64 rows from position 0, heads of 64, 234 against 226, the
+//   same from 30 235 against 237; heads of 128, 96 rows from 0 277 against 269, 128 rows 292 against 296;
+//   more keys than attn_rows_kernel holds, where its two substitutes spread a row's keys over
+//   workgroups: 16 rows from 3500, heads of 64, 535 against 386, 32 rows 542 against 563; heads of
+//   32, 16 rows from 5500 522 against 505, 32 rows 528 against 806.
+// Otherwise the flash kernel: 4 rows from 2000, heads of 64, 362 against 708.
+inline bool takes_flash(bool exact, int D, int n, int kmax, bool rows_fit)
+{
+    if (exact || kmax <= (D == 128 ? 112 : 64)) return false;
+    return rows_fit || n >= kFlashRows;
 }
 
 // The exact-order attention of one query head for kWeighDims value dimensions (the reference's
@@ -1217,12 +1484,15 @@ int prefill_layer(fg_qwen2 *m, size_t li, size_t first, int n, hipStream_t st)
     a.corr = m->pre.lco;
     a.row_width = width;
     const int D = int(sh.head_dim), kmax = int(first) + n;
-    if (const size_t rsmem = attn_rows_smem(D, kmax)) {
+    a.rope = m->rope;
+    a.kkeep = m->kcache;
+    a.vkeep = m->vcache;
+    const size_t rsmem = attn_rows_smem(D, kmax);
+    if (takes_flash(sh.exact, D, n, kmax, rsmem != 0)) {
+        if ((rc = D == 32 ? launch_flash<32>(a, n, st) : D == 64 ? launch_flash<64>(a, n, st) : launch_flash<128>(a, n, st))) return rc;
+    } else if (rsmem) {
         // blocks of rows sharing their keys and values (each row over its own keys), the chunk's
         // rows rotated and kept on the way
-        a.rope = m->rope;
-        a.kkeep = m->kcache;
-        a.vkeep = m->vcache;
         const int R = kAttnThreads / D;
         const dim3 rgrid(unsigned(sh.heads), unsigned((n + R - 1) / R));
         if (sh.exact) attn_rows_kernel<true><<<rgrid, kAttnThreads, rsmem, st>>>(a, n, (kmax + 3) / 4 * 4);
