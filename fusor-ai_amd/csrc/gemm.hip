@@ -1700,6 +1700,138 @@ __global__ __launch_bounds__(64) void t2_gemm_kernel(T2Params p)
     }
 }
 
+// T2b128 products of many tiles, staged: a workgroup of four waves owns 64 rows x 128 columns, wave w
+// the 32 x 64 at (w / 2, w % 2) as two 32 x 32 MFMA tiles. A stage is one group of 128 inputs: the
+// rows' levels [row][128], the columns' codes [quad][128], the rows' scales and corrections and
+// the columns' scales arrive by direct global-to-LDS loads (whole runs of memory by neighbouring
+// lanes), three stages in turn, so a wave waits for loads issued two stages before. The 16-byte
+// pieces of a row (or quad) lie at their index xor the row's (quad's) low three bits, which
+// spreads a wave's operand reads over the banks. The group's dots start from the rows' corrections
+// and the rescale is t2_gemm_kernel's.
+// Bound: per 32 x 32 tile and group, 144 cycles of int8 MFMA and about 240 of VALU issue (the exact
+// rescale and the codes' unpacking): 40 us for 512 rows x 4096 -> 14336, measured 65 against 116 for
+// t2_gemm_kernel, whose waves read their operands from L2 a lane's row at a time.
+constexpr int kT2Rows = 64, kT2Cols = 128, kT2Stages = 3;
+constexpr int kT2LevelBytes = kT2Rows * 128, kT2CodeBytes = kT2Cols / 4 * 128;
+constexpr int kT2StageBytes = kT2LevelBytes + kT2CodeBytes + kT2Rows * 8 + kT2Cols * 4;
+
+template <bool FUSED>
+__global__ __launch_bounds__(256, 4) void t2_lds_kernel(T2Params p)
+{
+    extern __shared__ __align__(16) unsigned char t2_stage[];  // [kT2Stages][kT2StageBytes]
+    const int G = p.G, K = p.K;
+    const int tid = threadIdx.x, lane = tid & 63, i = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ncol = (p.quad_end - p.quad_begin) * 4, col_begin = p.quad_begin * 4;
+    int tx, ty;
+    tile_of(int(blockIdx.x), (ncol + kT2Cols - 1) / kT2Cols, (p.rows + kT2Rows - 1) / kT2Rows, tx, ty);
+    const int m0 = ty * kT2Rows, n0 = col_begin + tx * kT2Cols;
+
+    // this lane's addresses at group 0 (rows and columns past the edges re-read the last valid one)
+    const int8_t *level_src[2];
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        const int r = (2 * wave + t) * 8 + (lane >> 3);
+        level_src[t] = p.q + size_t(min(m0 + r, p.rows - 1)) * K + ((lane ^ r) & 7) * 16;
+    }
+    const int quad = wave * 8 + (lane >> 3);
+    const uint8_t *code_src = p.codes + size_t(min(n0 / 4 + quad, p.quad_end - 1)) * p.B * 32 + ((lane ^ quad) & 7) * 16;
+    const size_t row_at = size_t(min(m0 + lane, p.rows - 1)) * G;
+    const float *row_src = wave == 0 ? p.as + row_at : reinterpret_cast<const float *>(p.corr) + row_at;
+    const float *col_src = p.wscales + size_t(min(n0 / 4 + i, p.quad_end - 1)) * G * 4;
+    auto issue = [&](int g, int buf) {
+        unsigned char *base = t2_stage + buf * kT2StageBytes;
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const int8_t *src = level_src[t] + size_t(g) * 128;
+            __builtin_amdgcn_global_load_lds(src, base + (2 * wave + t) * 1024, 16, 0, 0);
+        }
+        const uint8_t *codes = code_src + size_t(g) * 128;
+        __builtin_amdgcn_global_load_lds(codes, base + kT2LevelBytes + wave * 1024, 16, 0, 0);
+        if (wave < 2) {  // a row's scale (wave 0) or correction (wave 1) per lane
+            const float *src = row_src + g;
+            __builtin_amdgcn_global_load_lds(src, base + kT2LevelBytes + kT2CodeBytes + wave * kT2Rows * 4, 4, 0, 0);
+        } else if (wave == 2 && h == 0) {  // a quad's four scales per lane
+            const float *src = col_src + size_t(g) * 4;
+            __builtin_amdgcn_global_load_lds(src, base + kT2LevelBytes + kT2CodeBytes + kT2Rows * 8, 16, 0, 0);
+        }
+    };
+    const int wr = 32 * (wave >> 1), wc = 64 * (wave & 1);
+    const int row = wr + i, sh = 4 * h;
+    float acc[2][16];
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[t][v] = 0.0f;
+
+    issue(0, 0);
+    if (G > 1) issue(1, 1);
+    int buf = 0;
+    for (int g = 0; g < G; g++) {
+        // this wave's loads of group g; those of group g + 1 (three, or four) stay in flight
+        if (g + 1 >= G) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        else if (wave == 3) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        stage_barrier();  // every wave's loads of group g; every wave done with group g - 1
+        if (g + 2 < G) issue(g + 2, buf >= 1 ? buf - 1 : 2);
+        const unsigned char *base = t2_stage + buf * kT2StageBytes;
+        const unsigned char *codes = base + kT2LevelBytes;
+        const float *row_scales = reinterpret_cast<const float *>(codes + kT2CodeBytes);
+        const int *row_corr = reinterpret_cast<const int *>(row_scales + kT2Rows);
+        const float *col_scales = reinterpret_cast<const float *>(row_corr + kT2Rows);
+        v4i a[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) a[k] = *reinterpret_cast<const v4i *>(base + row * 128 + (((2 * k + h) ^ row) & 7) * 16);
+        v16i start;  // the corrections, offset so that a total becomes a float by subtraction
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const v4i c = *reinterpret_cast<const v4i *>(row_corr + wr + 8 * j + 4 * h);
+#pragma unroll
+            for (int e = 0; e < 4; e++) start[4 * j + e] = c[e] + 0x4B400000;
+        }
+        v16i d[2];
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const int col = wc + 32 * t + i, q = col >> 2;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int2 w8 = *reinterpret_cast<const int2 *>(codes + q * 128 + (((2 * k + ((col >> 1) & 1)) ^ q) & 7) * 16 + (col & 1) * 8);
+                const int lo = w8.x >> sh, hi = w8.y >> sh;
+                const v4i w = {lo & 0x03030303, hi & 0x03030303, (lo >> 2) & 0x03030303, (hi >> 2) & 0x03030303};
+                d[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[k], w, k == 0 ? start : d[t], 0, 0, 0);
+            }
+        }
+        const float ws[2] = {col_scales[wc + i], col_scales[wc + 32 + i]};
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const v4f sc = *reinterpret_cast<const v4f *>(row_scales + wr + 8 * j + 4 * h);
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int v = 4 * j + e;
+                    const float D = unbiased(d[t][v]);
+                    acc[t][v] = FUSED ? __builtin_fmaf(D, ws[t] * sc[e], acc[t][v]) : acc[t][v] + D * (ws[t] * sc[e]);
+                }
+        }
+        buf = buf == 2 ? 0 : buf + 1;
+    }
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        const int n = n0 + wc + 32 * t + i;
+        if (n >= col_begin + ncol) continue;
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            const int r = m0 + wr + 8 * (v >> 2) + 4 * h + (v & 3);
+            if (r >= p.rows) continue;
+            float y = acc[t][v];
+            if (p.bias && n < p.n_rows) y = y + p.bias[n];
+            float *o = p.out + size_t(r) * p.ld_out + (n - col_begin);
+            *o = p.accumulate ? *o + y : y;
+        }
+    }
+}
+
 template <int TN, bool FUSED>
 int launch_t2_gemm_as(const T2Params &p, hipStream_t s)
 {
@@ -1709,11 +1841,23 @@ int launch_t2_gemm_as(const T2Params &p, hipStream_t s)
     return FG_OK;
 }
 
-// 32 x 64 tiles while they still give every SIMD two waves, else 32 x 32
+// The staged tiles from about a workgroup per CU, where their traffic and not one workgroup's chain
+// of stages (1 us a group) is what counts: 4096 x 14336 at 96 rows (224 workgroups) 36 us against 40,
+// 1024 x 4096 at 512 rows (256) 13.1 against 18.8, at 256 rows (128) 12.5 against 10.8, 896 x 4864 at
+// 256 rows (152) 11.4 against 11.7, 4864 x 896 at 1024 rows (112) 48 against 29. 32 rows would leave
+// half of each tile empty: they keep one wave per tile of 32 x 64 while that gives every SIMD two
+// waves, else 32 x 32.
+constexpr long kT2StagedGroups = 200;
 template <bool FUSED>
 int launch_t2_gemm(const T2Params &p, hipStream_t s)
 {
     const long wide = long((p.quad_end - p.quad_begin) * 4 + 63) / 64 * ((p.rows + 31) / 32);
+    const long staged = long((p.quad_end - p.quad_begin) * 4 + kT2Cols - 1) / kT2Cols * ((p.rows + kT2Rows - 1) / kT2Rows);
+    if (p.rows > 32 && staged >= kT2StagedGroups) {
+        t2_lds_kernel<FUSED><<<unsigned(staged), 256, kT2Stages * kT2StageBytes, s>>>(p);
+        FG_HIP(hipGetLastError());
+        return FG_OK;
+    }
     return wide >= kT2WideTiles ? launch_t2_gemm_as<2, FUSED>(p, s) : launch_t2_gemm_as<1, FUSED>(p, s);
 }
 
