@@ -134,8 +134,13 @@ def check(rc):
 def stream_handle(stream=None):
     """The hipStream_t of `stream` (torch's current stream by default)."""
     import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    if stream is not None:
+        return ctypes.c_void_p(stream.cuda_stream)
+    # the current stream's handle itself: torch.cuda.current_stream() looks its device up through
+    # torch.device and builds a Stream around the handle, about 3 us of a call's 10
+    if torch.cuda.is_initialized():
+        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
+    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
 def ptr(t):
