@@ -1782,12 +1782,12 @@ __global__ __launch_bounds__(256, 4) void t2_lds_kernel(T2Params p)
         v4i a[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) a[k] = *reinterpret_cast<const v4i *>(base + row * 128 + (((2 * k + h) ^ row) & 7) * 16);
-        v16i start;  // the corrections, offset so that a total becomes a float by subtraction
+        v16i start;  // the rows' corrections: the dots start from them
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const v4i c = *reinterpret_cast<const v4i *>(row_corr + wr + 8 * j + 4 * h);
 #pragma unroll
-            for (int e = 0; e < 4; e++) start[4 * j + e] = c[e] + 0x4B400000;
+            for (int e = 0; e < 4; e++) start[4 * j + e] = c[e];
         }
         v16i d[2];
 #pragma unroll
@@ -1810,7 +1810,7 @@ __global__ __launch_bounds__(256, 4) void t2_lds_kernel(T2Params p)
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     const int v = 4 * j + e;
-                    const float D = unbiased(d[t][v]);
+                    const float D = float(d[t][v]);
                     acc[t][v] = FUSED ? __builtin_fmaf(D, ws[t] * sc[e], acc[t][v]) : acc[t][v] + D * (ws[t] * sc[e]);
                 }
         }
