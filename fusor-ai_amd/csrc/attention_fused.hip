@@ -24,7 +24,7 @@
 //
 // Bound: instruction issue. Additions and multiplications take 2.4 cycles a wave with two waves on the
 // SIMD, fused multiply-adds, maxima and byte permutes 4.2, so totals are converted by subtraction
-// (unbiased) and exponents taken from an addition's low bits (ref_exp): 4096 x 4096, 16 heads of
+// (unbiased) and exponents taken from an addition's low bits (exp_by_additions): 4096 x 4096, 16 heads of
 // 72, in 321 us (409 with conversion instructions), 365 a call with the keys' and values'
 // preparation, against 941 unit by unit. 16 queries a wave (16 x 16 products, four waves a SIMD)
 // take 530 us: the same arithmetic with twice the instructions around it.
@@ -217,6 +217,36 @@ __global__ __launch_bounds__(256) void key_record_kernel(FusedParams p, unsigned
     const unsigned half = sub / 4;
     *reinterpret_cast<int *>(rec + b * 1024 + (half * 32 + key) * 16 + (sub & 3) * 4) = live ? packed : 0;
     if (sub == 0) *reinterpret_cast<float *>(rec + R::kKeyScales + b * 128 + key * 4) = live ? d : 0.0f;
+}
+
+// ref_exp and ref_exp_fast by additions: that of 1.5 · 2^23 rounds to an integer, ties to even, and
+// leaves it in the low bits, where rint, the conversion and the shifted sum issue at half the rate.
+// Same bits; a longer chain, so not for kernels of one wave a SIMD.
+template <bool FAST>
+__device__ __forceinline__ float exp_by_additions(float x)
+{
+    x = FAST ? fmaxf(x, -87.0f) : x < -87.0f ? -87.0f : (x > 88.0f ? 88.0f : x);
+    const float rounded = x * 1.44269504088896340736f + 12582912.0f;
+    const float n = rounded - 12582912.0f;
+    float poly;
+    if (FAST) {
+        const float r = __builtin_fmaf(-n, 0.693147180559945309417f, x);
+        poly = 1.0f / 24.0f;
+        poly = __builtin_fmaf(poly, r, 1.0f / 6.0f);
+        poly = __builtin_fmaf(poly, r, 0.5f);
+        poly = __builtin_fmaf(poly, r, 1.0f);
+        poly = __builtin_fmaf(poly, r, 1.0f);
+    } else {
+        const float r = x - n * 0.6933594f - n * -2.1219444e-4f;
+        poly = 1.9875691e-4f;
+        poly = poly * r + 1.3981999e-3f;
+        poly = poly * r + 8.333452e-3f;
+        poly = poly * r + 4.1665796e-2f;
+        poly = poly * r + 0.16666666f;
+        poly = poly * r + 0.5f;
+        poly = poly * r * r + r + 1.0f;
+    }
+    return poly * __uint_as_float((__float_as_uint(rounded) << 23) + 0x3F800000u);
 }
 
 // The low bytes of four dwords as one.
@@ -414,7 +444,7 @@ __global__ __launch_bounds__(256, 2) void attend_fused_kernel(FusedParams p)
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const float x = s[n][r] * p.scale - peak;
-                s[n][r] = FAST ? ref_exp_fast(x) : ref_exp(x);
+                s[n][r] = exp_by_additions<FAST>(x);
                 if (MASKED && 8 * (r / 4) + 4 * half + r % 4 >= left) s[n][r] = 0.0f;
             }
 #pragma unroll

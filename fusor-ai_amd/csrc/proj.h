@@ -119,21 +119,12 @@ __host__ __device__ inline ProjLayout proj_layout(int R, int K, int G, int NW, i
     return l;
 }
 
-// 2^n from the bits of 1.5 · 2^23 + n, n in [-126, 127].
-__device__ __forceinline__ float exp_scale(float rounded)
-{
-    return __uint_as_float((__float_as_uint(rounded) << 23) + 0x3F800000u);
-}
-
 // ops::exp (ops.rs:97-131): clamp, n = round(x·log2 e), r = x − n·ln2_hi − n·ln2_lo, Cephes
 // polynomial in Horner order, times 2^n through the exponent bits. No fused multiply-add.
 __device__ __forceinline__ float ref_exp(float x)
 {
     x = x < -87.0f ? -87.0f : (x > 88.0f ? 88.0f : x);
-    // the addition of 1.5 · 2^23 rounds to an integer, ties to even, and leaves it in the low bits:
-    // rint, the conversion and ldexp issue at half the rate of these additions and the multiplication
-    const float rounded = x * 1.44269504088896340736f + 12582912.0f;
-    const float exponent = rounded - 12582912.0f;
+    const float exponent = __builtin_rintf(x * 1.44269504088896340736f);
     const float remainder = x - exponent * 0.6933594f - exponent * -2.1219444e-4f;
     float poly = 1.9875691e-4f;
     poly = poly * remainder + 1.3981999e-3f;
@@ -142,7 +133,8 @@ __device__ __forceinline__ float ref_exp(float x)
     poly = poly * remainder + 0.16666666f;
     poly = poly * remainder + 0.5f;
     poly = poly * remainder * remainder + remainder + 1.0f;
-    return poly * exp_scale(rounded);
+    const int bits = (int(exponent) + 127) << 23;
+    return poly * __int_as_float(bits);
 }
 
 // exp_fast (ops.rs:137-153): clamped below at EXP_MIN, n = round(x · log2 e) ties to even,
@@ -150,15 +142,14 @@ __device__ __forceinline__ float ref_exp(float x)
 __device__ __forceinline__ float ref_exp_fast(float x)
 {
     x = fmaxf(x, -87.0f);
-    const float rounded = x * 1.44269504088896340736f + 12582912.0f;  // as in ref_exp
-    const float n = rounded - 12582912.0f;
+    const float n = rintf(x * 1.44269504088896340736f);
     const float r = __builtin_fmaf(-n, 0.693147180559945309417f, x);
     float poly = 1.0f / 24.0f;
     poly = __builtin_fmaf(poly, r, 1.0f / 6.0f);
     poly = __builtin_fmaf(poly, r, 0.5f);
     poly = __builtin_fmaf(poly, r, 1.0f);
     poly = __builtin_fmaf(poly, r, 1.0f);
-    return poly * exp_scale(rounded);
+    return poly * __int_as_float((int(n) + 127) << 23);
 }
 
 // ops::silu (ops.rs:272-274)
