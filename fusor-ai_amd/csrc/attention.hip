@@ -15,6 +15,8 @@
 // accumulators and the reference's f32 group order. The f32 steps around them follow the
 // reference's order: the mean is a sequential sum per channel, the exponentials' sum is the
 // scalar backend's (eight offset sums over whole runs of eight, then the rest and those sums).
+// This is the step-by-step path, a head's scores in memory: heads past 128, and few rows over many
+// keys (takes_fused). The rest run in attention_fused.hip.
 #include "attention.h"
 #include "common.h"
 #include "proj.h"
@@ -31,6 +33,21 @@ constexpr int kMaxRowBytes = 64 * 1024;  // one padded score row in LDS: at most
 constexpr int kMaxHeadDim = 1024;
 
 size_t pad32(size_t n) { return (n + 31) / 32 * 32; }
+
+// exp_fast (ops.rs:137-153): clamped below at EXP_MIN, n = round(x · log2 e) ties to even,
+// r = fma(−n, ln 2, x), the degree-4 Taylor polynomial in fused multiply-adds, times 2^n.
+__device__ __forceinline__ float ref_exp_fast(float x)
+{
+    x = fmaxf(x, -87.0f);
+    const float n = rintf(x * 1.44269504088896340736f);
+    const float r = __builtin_fmaf(-n, 0.693147180559945309417f, x);
+    float poly = 1.0f / 24.0f;
+    poly = __builtin_fmaf(poly, r, 1.0f / 6.0f);
+    poly = __builtin_fmaf(poly, r, 0.5f);
+    poly = __builtin_fmaf(poly, r, 1.0f);
+    poly = __builtin_fmaf(poly, r, 1.0f);
+    return poly * __int_as_float((int(n) + 127) << 23);
+}
 
 // keyT[(t · hd + d) · kpad + k] = key[k][d] of table t = image · kv_heads + kh: the keys of every
 // (image, key head) with channels as rows, through 64 x 64 tiles in LDS (both sides coalesced).

@@ -137,21 +137,6 @@ __device__ __forceinline__ float ref_exp(float x)
     return poly * __int_as_float(bits);
 }
 
-// exp_fast (ops.rs:137-153): clamped below at EXP_MIN, n = round(x · log2 e) ties to even,
-// r = fma(−n, ln 2, x), the degree-4 Taylor polynomial in fused multiply-adds, times 2^n.
-__device__ __forceinline__ float ref_exp_fast(float x)
-{
-    x = fmaxf(x, -87.0f);
-    const float n = rintf(x * 1.44269504088896340736f);
-    const float r = __builtin_fmaf(-n, 0.693147180559945309417f, x);
-    float poly = 1.0f / 24.0f;
-    poly = __builtin_fmaf(poly, r, 1.0f / 6.0f);
-    poly = __builtin_fmaf(poly, r, 0.5f);
-    poly = __builtin_fmaf(poly, r, 1.0f);
-    poly = __builtin_fmaf(poly, r, 1.0f);
-    return poly * __int_as_float((int(n) + 127) << 23);
-}
-
 // ops::silu (ops.rs:272-274)
 __device__ __forceinline__ float ref_silu(float x) { return x / (1.0f + ref_exp(-x)); }
 
