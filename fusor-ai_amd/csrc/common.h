@@ -104,6 +104,17 @@ __device__ __forceinline__ void stage_barrier()
     asm volatile("" ::: "memory");
 }
 
+// Orders a wave's LDS accesses around an exchange between its own lanes: what any lane wrote before
+// is read, and what any lane read before is overwritten, only after. The hardware keeps one wave's
+// LDS operations in order, so this emits nothing; without it the compiler, which reasons per lane,
+// may move a lane's read over a store of its own that it finds at another address.
+__device__ __forceinline__ void wave_exchange()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // The partner lane's value in pairs (lane ^ 1), through DPP.
 __device__ __forceinline__ int xor1(int v) { return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false); }
 // lane ^ 2 within a quad, and the mirror lane within 8 (lane ^ 7), through DPP.

@@ -670,7 +670,9 @@ __global__ __launch_bounds__(64 * kFlashWaves, 2) void attn_flash_kernel(AttnPar
         } else {
             load_keys(b);
         }
+        wave_exchange();  // the block before's keys are read
         store_keys();
+        wave_exchange();  // every lane's rows are written
         v16f s = {};
 #pragma unroll
         for (int c = 0; c < H / 4; c++) {
@@ -736,7 +738,8 @@ __global__ __launch_bounds__(64 * kFlashWaves, 2) void attn_flash_kernel(AttnPar
             }
         }
     }
-    // the waves' partial rows merged
+    // the waves' partial rows merged, each in its wave's part of the region
+    wave_exchange();  // the last block's keys are read
     {
         float *dst = part + (wave * kFlashRows + l31) * S;
 #pragma unroll
