@@ -15,9 +15,10 @@
 // accumulators and the reference's f32 group order. The f32 steps around them follow the
 // reference's order: the mean is a sequential sum per channel, the exponentials' sum is the
 // scalar backend's (eight offset sums over whole runs of eight, then the rest and those sums).
-// This is the step-by-step path, a head's scores in memory: heads past 128, and few rows over many
-// keys (takes_fused). The rest run in attention_fused.hip.
+// This is the step-by-step path, a head's scores in memory: heads past 128, few rows over many keys and
+// few heads (takes_fused). The rest run in attention_fused.hip.
 #include "attention.h"
+#include "attention_route.h"
 #include "common.h"
 #include "proj.h"
 
@@ -534,14 +535,7 @@ int run(const fg_attention *c, float *out, hipStream_t st, const Shape &s, const
     return FG_OK;
 }
 
-// Whether the call runs in the one launch of attention_fused.hip instead of a unit at a time. The
-// one launch walks a row's blocks of 32 keys in order, so few rows over many keys leave the chip
-// idle behind that chain; a unit at a time pays two launches per unit but spreads its keys. Both
-// sides as fitted, in microseconds, to measurements over 1 to 48 units, 1 to 1024 queries, 64 to
-// 16384 keys and heads of 32 to 128, of which the line misplaces those within about 20 % of it
-// (fast exponentials, heads of 64, one launch against unit by unit: 6 units x 1024 queries x 1024
-// keys 76 against 109; 1 unit of the same 75 against 56; 12 units x 1024 x 4096 256 against 371;
-// 12 units x 1 x 4096 249 against 210).
+// Whether the call runs in the one launch of attention_fused.hip instead of a unit at a time.
 bool takes_fused(const fg_attention *c)
 {
     // FG_ATTEND_UNITS sizes the step-by-step batches, so it asks for them
@@ -550,13 +544,8 @@ bool takes_fused(const fg_attention *c)
     const size_t tables = c->images * c->kv_heads, blocks = (c->keys + 31) / 32;
     const size_t lanes = std::max({tables * blocks * 32 * 8 * ((c->head_dim + 31) / 32), tables * blocks * (c->head_dim + 8),
                                    c->images * c->heads * ((c->queries + 127) / 128) * 256});
-    if (lanes >= (size_t(1) << 31)) return false;
-    const double units = double(c->images * c->heads), keys = double(c->keys), queries = double(c->queries);
-    const double hd = double(c->head_dim), waves = units * std::ceil(queries / 32);
-    const double block = 0.65 + 0.0215 * hd + (c->exponentials == FG_EXP_FAST ? 0.0 : 0.5);
-    const double fused = 20 + double(blocks) * block * std::max(1.0, 0.7 * waves / 1024);
-    const double steps = 45 + 6.6 * units + 1.2e-4 * keys * hd + units * keys * (0.00115 + 3.5e-6 * queries);
-    return fused <= steps;
+    return lanes < (size_t(1) << 31) &&
+           attend_in_one_launch(c->images, c->heads, c->head_dim, c->queries, c->keys, c->exponentials == FG_EXP_FAST);
 }
 
 }  // namespace
