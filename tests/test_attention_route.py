@@ -43,3 +43,9 @@ def rule(tmp_path_factory):
 def test_the_faster_path(rule, call):
     head_dim, images, heads, queries, keys, fast, launch, steps = call
     assert rule(images, heads, head_dim, queries, keys, fast) == (launch < steps)
+
+
+def test_the_one_launch_tests_take_the_one_launch(rule):
+    from test_gpu_attention_fused import LONG, RECORDS, SHAPES
+    for H, _, D, I, Q, K, fast in SHAPES + RECORDS + LONG:
+        assert rule(I, H, D, Q, K, fast), (H, D, I, Q, K, fast)

@@ -1,9 +1,10 @@
 """fg_attend (attention::attend, blocks/src/attention.rs:81-214) on the GPU against the oracle.
 
 Every step is deterministic and the f32 steps follow the reference's order, so the outputs are
-bit-identical to the oracle's for both exponentials, across the product's row paths (1-4 rows
-on the matrix-vector kernel, 5-16 and 17+ on the matrix cores), grouped heads, several images,
-padded head and key counts, and operands read by stride and offset from one fused row."""
+bit-identical to the oracle's for both exponentials, grouped heads, several images, padded head and
+key counts, and operands read by stride and offset from one fused row; and unit by unit
+(FG_ATTEND_UNITS asks for it) across the product's row paths (1-4 rows on the matrix-vector
+kernel, 5-16 and 17+ on the matrix cores)."""
 import numpy as np
 import pytest
 
@@ -46,6 +47,8 @@ def same_bits(a, b):
     return a.shape == b.shape and np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
+# the comments name the kernels unit by unit; a call by itself takes the shapes of up to 300 keys in
+# one launch, the four of 1000 keys and more stay unit by unit
 CASES = [  # heads, kv_heads, head_dim, images, queries, keys, fast
     (2, 2, 64, 1, 3, 200, True),      # 3 query rows: the scores on the matrix-vector kernel
     (6, 1, 32, 3, 5, 9, True),        # 5 rows: the scores on the 16-row matrix-core kernel
@@ -71,6 +74,12 @@ def test_attend_is_the_oracles_bits(fk, case):
     want = O.attend(H, KV, D, I, Q, K, q, k, v, fast=fast)
     got = gpu_attend(fk, H, KV, D, I, Q, K, q, k, v, fast)
     assert same_bits(got, want), np.max(np.abs(got - want))
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_attend_unit_by_unit_is_the_oracles_bits(fk, monkeypatch, case):
+    monkeypatch.setenv("FG_ATTEND_UNITS", "64")
+    test_attend_is_the_oracles_bits(fk, case)
 
 
 @pytest.mark.parametrize("units", [1, 4, 5])
