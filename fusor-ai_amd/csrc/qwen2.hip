@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "common.h"
+#include "prefill_route.h"
 #include "proj.h"
 
 namespace fg {
@@ -830,20 +831,6 @@ inline size_t attn_rows_smem(int D, int kmax)
     return bytes <= 64 * 1024 ? bytes : 0;
 }
 
-// Which kernels a chunk of n rows whose last sees kmax keys takes, in parallel order (head sizes are
-// 32, 64 or 128). Four layers' reads with attn_flash_kernel against the others, microseconds:
-//   few keys, one launch instead of two: 64 rows from position 0, heads of 64, 234 against 226, the
-//   same from 30 235 against 237; heads of 128, 96 rows from 0 277 against 269, 128 rows 292 against 296;
-//   more keys than attn_rows_kernel holds, where its two substitutes spread a row's keys over
-//   workgroups: 16 rows from 3500, heads of 64, 535 against 386, 32 rows 542 against 563; heads of
-//   32, 16 rows from 5500 522 against 505, 32 rows 528 against 806.
-// Otherwise the flash kernel: 4 rows from 2000, heads of 64, 362 against 708.
-inline bool takes_flash(bool exact, int D, int n, int kmax, bool rows_fit)
-{
-    if (exact || kmax <= (D == 128 ? 112 : 64)) return false;
-    return rows_fit || n >= kFlashRows;
-}
-
 // The exact-order attention of one query head for kWeighDims value dimensions (the reference's
 // arithmetic of attn_weigh_kernel<true>, ops.rs:301-342), over the scores of the cached keys that
 // the query launch formed (score_chunk). Grid: (heads, D / kWeighDims), 256 threads.
@@ -1491,7 +1478,7 @@ int prefill_layer(fg_qwen2 *m, size_t li, size_t first, int n, hipStream_t st)
     a.kkeep = m->kcache;
     a.vkeep = m->vcache;
     const size_t rsmem = attn_rows_smem(D, kmax);
-    if (takes_flash(sh.exact, D, n, kmax, rsmem != 0)) {
+    if (!sh.exact && prefill_takes_flash(D, a.heads, a.kv_heads, n, kmax, rsmem != 0)) {
         if ((rc = D == 32 ? launch_flash<32>(a, n, st) : D == 64 ? launch_flash<64>(a, n, st) : launch_flash<128>(a, n, st))) return rc;
     } else if (rsmem) {
         // blocks of rows sharing their keys and values (each row over its own keys), the chunk's

@@ -23,7 +23,7 @@ pytestmark = pytest.mark.gpu
 LIMIT = 1.3e-2
 
 HIDDEN, FFN = 128, 32
-SEED = 107  # inputs in which every planted mistake moves some row by 4e-2 or more
+SEED = 112  # inputs in which every planted mistake moves some row by 3.7e-2 or more
 HEADS = {32: (6, 3), 64: (4, 1), 128: (2, 2)}
 
 
@@ -78,10 +78,11 @@ def read_caches(fk, params, embeddings, first, chunk, exact):
     return [t.cpu().numpy()[1, :, first:first + n] for t in (kd, vd)]
 
 
-# more than 64 keys (112 for heads of 128), or the kernel for few keys takes the chunk
-SHAPES = [(1, 112), (31, 82), (32, 96), (33, 95), (65, 63), (129, 0), (40, 255), (33, 700)]
+# few keys stay with attn_rows_kernel: up to 64 (heads of 128: 112), of fewer than 32 rows up to
+# 144 (160)
+SHAPES = [(1, 160), (7, 158), (31, 130), (32, 96), (33, 95), (65, 63), (129, 0), (40, 255), (33, 700)]
 # past 1484, 2988 and 5996 keys (heads of 32, 64, 128) attn_rows_kernel does not hold a block's scores
-LONG = [(32, 33, 1480), (64, 64, 3000), (128, 32, 6000)]
+LONG = [(32, 48, 1480), (64, 110, 2900), (128, 180, 5850)]
 CASES = [(d, *s) for d in (32, 64, 128) for s in SHAPES] + LONG
 
 
