@@ -16,6 +16,7 @@
 // K positions are used for both operands, so the sum covers the block's 32 inputs. Result:
 // lane l holds column l % 32, rows 8·(v/4) + 4·(l/32) + v%4 for v = 0..15.
 #include "common.h"
+#include "t2_route.h"
 
 #include <cstdint>
 #include <cstdlib>
@@ -1711,7 +1712,7 @@ __global__ __launch_bounds__(64) void t2_gemm_kernel(T2Params p)
 // Bound: per 32 x 32 tile and group, 144 cycles of int8 MFMA and about 240 of VALU issue (the exact
 // rescale and the codes' unpacking): 40 us for 512 rows x 4096 -> 14336, measured 65 against 116 for
 // t2_gemm_kernel, whose waves read their operands from L2 a lane's row at a time.
-constexpr int kT2Rows = 64, kT2Cols = 128, kT2Stages = 3;
+constexpr int kT2Stages = 3;
 constexpr int kT2LevelBytes = kT2Rows * 128, kT2CodeBytes = kT2Cols / 4 * 128;
 constexpr int kT2StageBytes = kT2LevelBytes + kT2CodeBytes + kT2Rows * 8 + kT2Cols * 4;
 
@@ -1841,20 +1842,14 @@ int launch_t2_gemm_as(const T2Params &p, hipStream_t s)
     return FG_OK;
 }
 
-// The staged tiles from about a workgroup per CU, where their traffic and not one workgroup's chain
-// of stages (1 us a group) is what counts: 4096 x 14336 at 96 rows (224 workgroups) 36 us against 40,
-// 1024 x 4096 at 512 rows (256) 13.1 against 18.8, at 256 rows (128) 12.5 against 10.8, 896 x 4864 at
-// 256 rows (152) 11.4 against 11.7, 4864 x 896 at 1024 rows (112) 48 against 29. 32 rows would leave
-// half of each tile empty: they keep one wave per tile of 32 x 64 while that gives every SIMD two
-// waves, else 32 x 32.
-constexpr long kT2StagedGroups = 200;
+// The staged tiles where t2_takes_staged has them, else one wave per tile of 32 x 64 while that gives every
+// SIMD two waves, else of 32 x 32.
 template <bool FUSED>
 int launch_t2_gemm(const T2Params &p, hipStream_t s)
 {
-    const long wide = long((p.quad_end - p.quad_begin) * 4 + 63) / 64 * ((p.rows + 31) / 32);
-    const long staged = long((p.quad_end - p.quad_begin) * 4 + kT2Cols - 1) / kT2Cols * ((p.rows + kT2Rows - 1) / kT2Rows);
-    if (p.rows > 32 && staged >= kT2StagedGroups) {
-        t2_lds_kernel<FUSED><<<unsigned(staged), 256, kT2Stages * kT2StageBytes, s>>>(p);
+    const long outputs = long(p.quad_end - p.quad_begin) * 4, wide = (outputs + 63) / 64 * ((p.rows + 31) / 32);
+    if (t2_takes_staged(p.rows, outputs, p.G)) {
+        t2_lds_kernel<FUSED><<<unsigned(t2_staged_groups(p.rows, outputs)), 256, kT2Stages * kT2StageBytes, s>>>(p);
         FG_HIP(hipGetLastError());
         return FG_OK;
     }

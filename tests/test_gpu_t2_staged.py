@@ -1,7 +1,7 @@
 """T2b128 products on the staged tiles (t2_lds_kernel: more than 32 rows, 200 or more workgroups of
 64 x 128), where their tiles, quads and three stage buffers end: 1 to 5 groups, row and column
-remainders, column ranges, bias, adding to the output, the fused scaling; and the 32 x 64 wave tiles that
-large tables of few rows keep. Every output is the oracle's bits."""
+remainders, column ranges, bias, adding to the output, the fused scaling; and the wave tiles that
+large tables of few rows, or of few past 64 and many groups, keep. Every output is the oracle's bits."""
 import numpy as np
 import pytest
 
@@ -13,8 +13,11 @@ pytestmark = pytest.mark.gpu
 
 
 # outputs are drawn so that ceil(rows / 64) * ceil(outputs / 128) >= 200 for the column range too
-@pytest.mark.parametrize("rows,outputs,groups", [(33, 25732, 1), (64, 25600, 2), (65, 12932, 3), (127, 12801, 4),
-                                                 (449, 3458, 5), (200, 6500, 3), (20, 131076, 1)])
+STAGED = [(33, 25732, 1), (64, 25600, 2), (65, 12932, 3), (127, 12801, 4), (449, 3458, 5), (200, 6500, 3)]
+WAVES = [(20, 131076, 1), (65, 12932, 9)]
+
+
+@pytest.mark.parametrize("rows,outputs,groups", STAGED + WAVES)
 def test_staged_t2_tiles(gpu, rows, outputs, groups):
     import fusor_kernels as fk
     import torch
