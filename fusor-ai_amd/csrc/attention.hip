@@ -583,7 +583,7 @@ extern "C" int fg_attend(const fg_attention *c, float *out, void *stream)
     Scratch w(s);
     void *ws = nullptr;
     FG_HIP(workspace_alloc(&ws, fused ? attend_fused_bytes(c) : w.total(), st));
-    w.carve(ws);
+    if (!fused) w.carve(ws);
     int rc = fused ? launch_attend_fused(c, out, ws, st) : run(c, out, st, s, w);
     // the scratch goes back to the pool in stream order, after the call's last kernel
     const hipError_t e = hipFreeAsync(ws, st);
