@@ -25,9 +25,10 @@
 // Bound: instruction issue. Additions and multiplications take 2.4 cycles a wave with two waves on the
 // SIMD, fused multiply-adds, maxima and byte permutes 4.2, so totals are converted by subtraction
 // (unbiased) and exponents taken from an addition's low bits (exp_by_additions): 4096 x 4096, 16 heads of
-// 72, in 321 us (409 with conversion instructions), 365 a call with the keys' and values'
-// preparation, against 941 unit by unit. 16 queries a wave (16 x 16 products, four waves a SIMD)
-// take 530 us: the same arithmetic with twice the instructions around it.
+// 72, in 342 us at its fastest dispatch and 369 on average, 365 a call with the keys' and values'
+// preparation in a loop of calls (452 with conversion instructions), against 941 unit by unit. 16 queries a
+// wave (16 x 16 products, four waves a SIMD) took 560 a call where 32 took 452: the same arithmetic with
+// twice the instructions around it.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>

@@ -1710,8 +1710,8 @@ __global__ __launch_bounds__(64) void t2_gemm_kernel(T2Params p)
 // spreads a wave's operand reads over the banks. The group's dots start from the rows' corrections
 // and the rescale is t2_gemm_kernel's.
 // Bound: per 32 x 32 tile and group, 144 cycles of int8 MFMA and about 240 of VALU issue (the exact
-// rescale and the codes' unpacking): 40 us for 512 rows x 4096 -> 14336, measured 65 against 116 for
-// t2_gemm_kernel, whose waves read their operands from L2 a lane's row at a time.
+// rescale and the codes' unpacking): 40 us for 512 rows x 4096 -> 14336, measured 71 on average (69 at its
+// fastest) against 128 for t2_gemm_kernel, whose waves read their operands from L2 a lane's row at a time.
 constexpr int kT2Stages = 3;
 constexpr int kT2LevelBytes = kT2Rows * 128, kT2CodeBytes = kT2Cols / 4 * 128;
 constexpr int kT2StageBytes = kT2LevelBytes + kT2CodeBytes + kT2Rows * 8 + kT2Cols * 4;

@@ -585,7 +585,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_rows_kernel(AttnParams a, i
 // Bound: the f32 matrix rate, 4096 cycles a block of 32 rows x 32 keys x 64 dimensions, beside about
 // 1300 of VALU work; with few blocks a wave, the chain of loads before and merge after them. 14 heads
 // of 64 over 2, 512 rows, after 0, 512 and 1024 others: 30 us a chunk on average where the VALU
-// kernel above (each row of the block reading every staged key and value) took 163; 158 rows 11.1
+// kernel above (each row of the block reading every staged key and value) took 163; 158 rows 11.3
 // and 3.2 for keep_rows_kernel where it took 17.5.
 // Error of the f32 rows against 64 bits, over chunks of 8 to 512 rows after 0 to 1300 others, caches of
 // unit and fourfold keys: 0.5 to 1.02 times attn_rows_kernel's and its substitutes' (heads of 64, 512 rows after
