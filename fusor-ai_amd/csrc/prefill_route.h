@@ -18,7 +18,10 @@ namespace fg {
 //   128 over 1, 1447 against 846; 64 rows from 5000, 4 heads of 64 over 4, 684 against 620, 96 rows 689
 //   against 922; 4 heads of 32 over 1, 32 rows from 7000 587 against 495. Under
 //   32 rows the substitutes are kept: 16 rows from 3500, heads of 64, 386 against 535.
-// Otherwise the flash kernel: 4 rows from 2000, heads of 64, 362 against 708.
+// Otherwise the flash kernel: 4 rows from 2000, heads of 64, 362 against 708. (5 to 16 rows of a model of 128
+// hidden values are bound by the host's launches, not by these kernels: up to about 450 keys the second launch is
+// their 7 %, 257 against 241. From 512 hidden values on the kernels are what counts: 8 rows over 160 keys, heads of 32,
+// 158 against 176, of 64 207 against 221, of 128 310 against 310.)
 inline bool prefill_takes_flash(int D, int heads, int kv_heads, int n, int kmax, bool rows_fit)
 {
     if (!rows_fit) return n >= 32 && (long long)n * (heads * D + 64 * kv_heads) >= 540ll * D;
